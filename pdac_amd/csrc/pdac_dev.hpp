@@ -71,7 +71,9 @@ struct Fields {
   double *snap_rgp, *snap_rlk;
   int32_t *ctr;                        // device counters (iter, ftem)
   unsigned long long *visits;          // work-list entries over all sweeps
-  int32_t *wl;                         // work list of one colour phase
+  int32_t *wl;                         // work lists of the colour phases: four of wlcap entries
+  long wlcap;
+  int32_t *team;                       // words of the iteration's team launches (TeamWord)
   // sweep flags (iter), one byte per cell in colour-major order (sweep_slot):
   // sdirty, the cell must be checked again; srefresh, the cell of the other
   // colour in the same pair changed in the previous phase and its snapshot

@@ -100,12 +100,19 @@ __device__ __forceinline__ void wl_append(int32_t *cnt, int32_t *list, bool pred
 }
 
 // device counters: sweep state of iter (done flag, sweep numbers of the two
-// colour launches, the sweep that converged, the first colour phase of the
-// call), EOS failures, three pairs of unconverged-cell counts per sweep
-// (C_WLP), and for the persistent iteration kernel an arrival counter for its
-// grid barriers and an error flag
-enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_PHB = 3, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
+// colour launches, the sweep that converged), EOS failures, three pairs of
+// unconverged-cell counts per sweep (C_WLP), and for the persistent iteration
+// kernels an arrival counter for grid barriers and an error flag
+enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
            C_ERR = 15, C_N = 16 };
+
+// Words of one team launch of the iteration (Fields::team, kTeamSlots of
+// them, cleared by k_predict): blocks of each XCD that have started, the XCD
+// chosen (+ 1; TL_NONE: none), the entries of the four cell lists, the
+// unconverged cells of three sweeps, and a barrier word per block.
+constexpr int kTeamBlocks = 32;  // blocks of a team: one per compute unit of an XCD
+constexpr int kTeamSlots = 8;    // team launches of one iter call
+enum TeamWord { TL_REG = 0, TL_STATE = 16, TL_CNT = 20, TL_UNC = 24, TL_BAR = 32, TL_STRIDE = 64, TL_NONE = 99 };
 
 // Whether the iteration of which the host has launched 'gate' sweeps has
 // ended, by the test the host applies after each batch of sweeps: a sweep
@@ -113,10 +120,12 @@ enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_PHB = 3, C_EOS = 4, C_NITF = 5, 
 // unconverged, or maxout sweeps ran.  The step's kernels after the
 // iteration are launched behind each batch with this gate, before the host
 // has read the batch's counters: they do nothing unless the batch ended the
-// iteration.  gate < 0: no gate.
+// iteration.  gate < 0: no gate; gate 0: only the done flag (behind a team
+// launch, which sets it whenever it ends the iteration).
 __device__ __forceinline__ bool iter_ended(const int32_t *ctr, int gate, int maxout) {
   if (gate < 0) return true;
   if (ctr[C_DONE]) return true;
+  if (gate == 0) return false;
   const int32_t *last = ctr + C_WLP + 2 * (gate % 3);
   if (last[0] + last[1] == 0) return true;
   return gate >= maxout;
@@ -1136,6 +1145,7 @@ __global__ void __launch_bounds__(kBlock, 3) k_tilde(Grid g, Consts K, Fields F,
 
 #include "pdac_visc.hip.inc"
 #include "pdac_iter.hip.inc"
+#include "pdac_team.hip.inc"
 #include "pdac_energy.hip.inc"
 #include "pdac_explicit.hip.inc"
 #include "pdac_ensemble.hip.inc"
