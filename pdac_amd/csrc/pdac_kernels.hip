@@ -106,13 +106,14 @@ __device__ __forceinline__ void wl_append(int32_t *cnt, int32_t *list, bool pred
 enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
            C_ERR = 15, C_N = 16 };
 
-// Words of one team launch of the iteration (Fields::team, kTeamSlots of
-// them, cleared by k_predict): blocks of each XCD that have started, the XCD
-// chosen (+ 1; TL_NONE: none), the entries of the four cell lists, the
-// unconverged cells of three sweeps, and a barrier word per block.
+// Words of the sweeps from lists (Fields::team, cleared by k_predict): the
+// lengths of k_visit's lists, and those of one team launch, cleared again
+// before the next: the lengths of its four lists, the blocks of each XCD that
+// have started, the XCD chosen (+ 1; TL_NONE: none), the unconverged cells of
+// three sweeps, and a barrier word per block.
 constexpr int kTeamBlocks = 32;  // blocks of a team: one per compute unit of an XCD
-constexpr int kTeamSlots = 8;    // team launches of one iter call
-enum TeamWord { TL_REG = 0, TL_STATE = 16, TL_CNT = 20, TL_UNC = 24, TL_BAR = 32, TL_STRIDE = 64, TL_NONE = 99 };
+enum TeamWord { TL_CNT = 0, TL_VIS = 8, TL_TEAM = 64, TL_REG = 64, TL_STATE = 80, TL_UNC = 84, TL_BAR = 96,
+                TL_TEAM_END = 128, TL_WORDS = 128, TL_NONE = 99 };
 
 // Whether the iteration of which the host has launched 'gate' sweeps has
 // ended, by the test the host applies after each batch of sweeps: a sweep
