@@ -1,7 +1,7 @@
-"""The explicit step's chain as a fixed point on the meshes that the 2D
-diagonal-major kernels do not take (3D, more than 512 columns, and
+"""The explicit step's chain as a fixed point (2D, 3D, ensembles and
 pdac_explicit_step_noalloc): equal bit for bit to the serial chain kernel
-(PDAC_CHAIN=general), whose order the reference's is."""
+(PDAC_CHAIN=general), whose order the reference's is, also where the iterates
+launched do not reach it and one work-group goes on (PDAC_CHAIN=1, 2)."""
 import ctypes as ct
 
 import numpy as np
@@ -40,12 +40,16 @@ CASES = {
 }
 
 
+def chain(monkeypatch, mode):
+    if mode is None:
+        monkeypatch.delenv("PDAC_CHAIN", raising=False)
+    else:
+        monkeypatch.setenv("PDAC_CHAIN", mode)
+
+
 def run(case, monkeypatch, general, noalloc=False, steps=4):
     from pdac_amd.gpu import gpu_solver, lib
-    if general:
-        monkeypatch.setenv("PDAC_CHAIN", "general")
-    else:
-        monkeypatch.delenv("PDAC_CHAIN", raising=False)
+    chain(monkeypatch, {True: "general", False: None}.get(general, general))
     g = gpu_solver(case, device=0)
     if noalloc:
         fail, cfl = ct.c_int32(), ct.c_double()
@@ -67,3 +71,37 @@ def test_fixed_point_equals_serial_chain(name, noalloc, monkeypatch):
     b = run(CASES[name](), monkeypatch, True)
     for k in b:
         np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+@pytest.mark.parametrize("iterates", ["1", "2"])
+@pytest.mark.parametrize("name", ["box_3d_3_classes", "wide_2d", "column_2d"])
+def test_one_work_group_goes_on(name, iterates, monkeypatch):
+    print(f"[chain fixed point] {name} after {iterates}", flush=True)
+    def case():
+        if name != "column_2d":
+            return CASES[name]()
+        c = eruption_column(nx=24, nz=40, dt=2.0e-4, vent_radius=6.0)
+        c.time_integration = 1
+        return c
+    a = run(case(), monkeypatch, iterates)
+    b = run(case(), monkeypatch, "general")
+    for k in b:
+        np.testing.assert_array_equal(a[k], b[k], err_msg=k)
+
+
+@pytest.mark.parametrize("mode", [None, "1"])
+def test_ensemble_of_3d_members(mode, monkeypatch):
+    from pdac_amd.gpu import Ensemble, gpu_solver
+    print(f"[chain fixed point] 3D ensemble {mode}", flush=True)
+    mk = lambda: [vent(), vent(), box(three_d=True, nx=9, ny=12, nz=5, nsolid=2)]
+    want = [run(c, monkeypatch, True, steps=3) for c in mk()]
+    chain(monkeypatch, mode)
+    ms = [gpu_solver(c, device=0) for c in mk()]
+    e = Ensemble(ms)
+    e.step(3)
+    for m, w in zip(ms, want):
+        got = m.state()
+        for k in got:
+            np.testing.assert_array_equal(got[k], w[k], err_msg=k)
+        m.close()
+    e.close()
