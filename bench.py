@@ -26,9 +26,8 @@ events on the dominant kernel, then steps on to --error-steps in all.
     python bench.py [--steps K] [--warmup W] [--gpus 1]
 
 Prints one JSON line with a "roofline" object for the dominant kernel
-(algorithmic bytes per launch over its mean HIP-event duration, with the
-HBM traffic rocprofv3 measured for it) and a "cpu_baseline" object (the CPU
-restatement of the same step, one core, on a bounded sample).
+(algorithmic bytes per launch over its mean HIP-event duration) and a
+"cpu_baseline" object (the CPU restatement of the same step, one core, on a bounded sample).
 """
 from __future__ import annotations
 
@@ -45,13 +44,6 @@ if ROOT not in sys.path:
     sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
-# HBM bytes per working launch of the sweep kernel (k_sweep, one colour
-# phase) on the default workload (FP32-flux form): rocprofv3 FETCH_SIZE and
-# WRITE_SIZE over its dispatches, each scaled by what the counter reads for a
-# copy of known size (--copy-calibration): 45.47 MB read + 6.55 MB written
-# over the 50,772 working dispatches of the default event region (steps
-# 260-360); None until measured
-SWEEP_TRAFFIC_PER_LAUNCH = 52.02e6
 # order of enum pdac_kernel (include/pdacgpu.h)
 KERNELS = ["boundary", "fieldn", "momflux", "tilde", "predict", "gasflux", "snapshot",
            "sweep", "ygas_flux", "ygas_update", "htilde_flux", "htilde_update", "ftem", "fill",
@@ -436,23 +428,23 @@ def main():
         dom, ms = "none", 0.0
     per_launch_s = ms / 1e3 / max(launches, 1) if launches else float("nan")
     traffic = None
-    if dom == "sweep":
-        # one launch is one colour phase of a sweep.  It reads the residual
-        # inputs of the cells whose inputs changed since their last check
-        # (check words) and runs the in-cell iteration, which reads and
-        # writes the reference sweep's words of a cell, for those not
-        # converged at visit start; the unchanged cells it skips would give
-        # the same result again.  Units counted on the device over the
-        # event region (pdac_profile_checks / pdac_profile_visits).
+    if dom in ("sweep", "iterate"):
+        # the kernels of the pressure-velocity iteration together: the checks
+        # and visits over the whole GPU ("sweep") and the team's sweeps
+        # ("iterate").  They read the residual inputs of the cells whose
+        # inputs changed since their last check (check words) and run the
+        # in-cell iteration, which reads and writes the reference sweep's
+        # words of a cell, for those not converged at visit start; the
+        # unchanged cells they skip would give the same result again.  Units
+        # counted on the device over the event region (pdac_profile_checks /
+        # pdac_profile_visits).
+        launches = prof["sweep"][0] + prof["iterate"][0]
+        per_launch_s = (prof["sweep"][1] + prof["iterate"][1]) / 1e3 / launches
+        dom = "sweep+iterate"
         checks, visits = r["checks"], r["visits"]
-        bytes_launch = 8.0 * ((checks - visits) * wc + visits * w["Is"]) / max(launches, 1)
-        if SWEEP_TRAFFIC_PER_LAUNCH is not None:
-            traffic = round(SWEEP_TRAFFIC_PER_LAUNCH)
-        unit_note = (f"per launch {checks / max(launches, 1):.0f} cells checked ({wc} words each) of which "
-                     f"{visits / max(launches, 1):.0f} visited ({w['Is']} words each)")
-    elif dom == "iterate":
-        bytes_launch = 8.0 * w["Is"] * n * sweeps_prof / max(launches, 1)
-        unit_note = f"ntot cells x sweeps per launch, {w['Is']} words per cell and sweep"
+        bytes_launch = 8.0 * ((checks - visits) * wc + visits * w["Is"]) / launches
+        unit_note = (f"per launch {checks / launches:.0f} cells checked ({wc} words each) of which "
+                     f"{visits / launches:.0f} visited ({w['Is']} words each)")
     elif dom == "none":
         bytes_launch, unit_note = 0.0, "kernel timing off"
     else:
