@@ -20,7 +20,7 @@ SOURCES = ["pdac_kernels.hip"]
 DEPS = ["pdac_kernels.hip", "pdac_iter.hip.inc", "pdac_team.hip.inc", "pdac_energy.hip.inc",
         "pdac_explicit.hip.inc", "pdac_ensemble.hip.inc", "pdac_api.hip.inc", "pdac_visc.hip.inc",
         "pdac_io.hip.inc", "pdac_setup.hip.inc",
-        "pdac_dev.hpp", "pdac_flux.hpp"]
+        "pdac_dev.hpp", "pdac_flux.hpp", "pdac_words.hpp"]
 ARCH = os.environ.get("PDAC_OFFLOAD_ARCH", "gfx950")
 
 FLAGS = [

@@ -19,6 +19,7 @@
 
 #include "pdac_dev.hpp"
 #include "pdac_flux.hpp"
+#include "pdac_words.hpp"
 
 using namespace pdac;
 
@@ -98,22 +99,6 @@ __device__ __forceinline__ void wl_append(int32_t *cnt, int32_t *list, bool pred
   base = __shfl(base, leader);
   if (pred) list[base + __popcll(m & ((1ull << lane) - 1ull))] = val;
 }
-
-// device counters: sweep state of iter (done flag, sweep numbers of the two
-// colour launches, the sweep that converged), EOS failures, three pairs of
-// unconverged-cell counts per sweep (C_WLP), and for the persistent iteration
-// kernels an arrival counter for grid barriers and an error flag
-enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
-           C_ERR = 15, C_N = 16 };
-
-// Words of the sweeps from lists (Fields::team, cleared by k_predict): the
-// lengths of k_visit's lists, and those of one team launch, cleared again
-// before the next: the lengths of its four lists, the blocks of each XCD that
-// have started, the XCD chosen (+ 1; TL_NONE: none), the unconverged cells of
-// three sweeps, and a barrier word per block.
-constexpr int kTeamBlocks = 32;  // blocks of a team: one per compute unit of an XCD
-enum TeamWord { TL_CNT = 0, TL_VIS = 8, TL_TEAM = 64, TL_REG = 64, TL_STATE = 80, TL_UNC = 84, TL_BAR = 96,
-                TL_TEAM_END = 128, TL_WORDS = 128, TL_NONE = 99 };
 
 // Whether the iteration of which the host has launched 'gate' sweeps has
 // ended, by the test the host applies after each batch of sweeps: a sweep
