@@ -1,9 +1,10 @@
-"""The team kernel of the pressure-velocity iteration (the sweeps after the
-first ones in one launch, from lists of the flagged cells) against one launch
-per colour phase: the cell arithmetic is the same and no order shows in the
+"""The team mode of the pressure-velocity iteration (whole-GPU checks and
+visits from lists while they are long, then the remaining sweeps in one
+launch) against one launch per colour phase: the cell arithmetic is the same and no order shows in the
 results, so every field and sweep count is equal bit for bit.  Small list
 limits make the team refuse, or stop at a sweep and launches go on from it;
 small maxout ends the iteration before it converges, inside either."""
+import ctypes as ct
 import os
 
 import numpy as np
@@ -24,22 +25,33 @@ CASES = {
     "box_2d_3_classes": lambda: mixed_box(nx=33, nz=21, nsolid=3, seed=5),
     "vent_odd": lambda: summit_vent_3d(nx=37, ny=41, nz=23, nsolid=2),
     "cone_40": lambda: summit_cone_3d(nx=40, ny=44, nz=30, height=230.0, sigma=230.0, rough=5.0),
+    # lists of a colour up to one round of the whole GPU's waves (2048 cells
+    # with three classes in 3D, 1024 with four, 8192 with one class in 2D) and
+    # beyond it
+    "box_one_round": lambda: mixed_box(three_d=True, nx=18, ny=18, nz=18, nsolid=3),
+    "box_over_a_round": lambda: mixed_box(three_d=True, nx=18, ny=18, nz=19, nsolid=3),
+    "box_4_classes_long": lambda: mixed_box(three_d=True, nx=17, ny=16, nz=15, nsolid=4, seed=7),
+    "box_2d_long": lambda: mixed_box(nx=140, nz=125, nsolid=1),
     "maxout_1": lambda: mixed_box(three_d=True, nx=10, ny=8, nz=9, nsolid=2, maxout=1),
     "maxout_3": lambda: mixed_box(nx=24, nz=18, nsolid=2, maxout=3),
 }
 
 
-def run(case, mode, limit=None, steps=3):
+def solver(case, **env):
     from pdac_amd.gpu import gpu_solver
-    env = {"PDAC_ITER_MODE": mode}
-    if limit:
-        env["PDAC_TEAM_LIMIT"] = str(limit)
     os.environ.update(env)
     try:
-        g = gpu_solver(case, device=0)
+        return gpu_solver(case, device=0)
     finally:
         for k in env:
             os.environ.pop(k)
+
+
+def run(case, mode, limit=None, steps=3):
+    env = {"PDAC_ITER_MODE": mode}
+    if limit:
+        env["PDAC_TEAM_LIMIT"] = str(limit)
+    g = solver(case, **env)
     nits = [g.step(1) for _ in range(steps)]
     nits.append(g.step_by_parts())
     out = {f.lower(): g.get(f.lower()) for f in abi.FIELDS}
@@ -58,3 +70,36 @@ def test_team_equals_launches(name, limit):
     assert a[0] == b[0] and a[1] == b[1], (a[:2], b[:2])
     bad = [k for k in b[2] if not np.array_equal(a[2][k], b[2][k], equal_nan=True)]
     assert not bad, bad
+
+
+# PDAC_K_YGAS_FLUX and PDAC_K_ITERATE (include/pdacgpu.h)
+K_YGAS_FLUX, K_ITERATE = 8, 15
+
+
+def launches(g, kernel):
+    n, ms = ct.c_int64(), ct.c_double()
+    assert g.lib.pdac_profile_read(g.ctx, kernel, ct.byref(n), ct.byref(ms)) == 0
+    return n.value
+
+
+def test_long_lists_take_few_attempts():
+    """Calls whose lists stay above the team's limit to the end, on a mesh
+    whose sweep grid counts as not resident: the sweeps go out in batches of
+    about as many as the last call took, so that a call makes a few attempts
+    at a team and not one per 16 sweeps, and the step's kernels behind the
+    iteration are launched once for the attempt that ends it and at most once
+    in vain."""
+    print("[team] long lists", flush=True)
+    g = solver(CASES["cone_40"](), PDAC_TEAM_LIMIT="1", PDAC_SWEEP_EARLY="0")
+    g.step(4)
+    g.lib.pdac_profile_select(g.ctx, (1 << K_YGAS_FLUX) | (1 << K_ITERATE))
+    g.lib.pdac_profile_enable(g.ctx, 1)
+    g.lib.pdac_profile_reset(g.ctx)
+    before, steps = g.nit_total, 16
+    g.step(steps)
+    sweeps, teams, ygas = g.nit_total - before, launches(g, K_ITERATE), launches(g, K_YGAS_FLUX)
+    g.close()
+    print(f"[team] {sweeps} sweeps, {teams} teams, {ygas} launches of the species fluxes in {steps} steps", flush=True)
+    assert sweeps > 40 * steps
+    assert teams <= 3 * steps
+    assert ygas <= 2 * steps
