@@ -105,3 +105,43 @@ def test_ensemble_of_3d_members(mode, monkeypatch):
             np.testing.assert_array_equal(got[k], w[k], err_msg=k)
         m.close()
     e.close()
+
+
+def test_pressures_that_are_not_numbers(monkeypatch):
+    """A state whose pressures have become NaN (its steps report the failure of
+    the equation of state): the iterates compare bits, so a NaN that stays is
+    no change, the stages are done after a few iterates again and the fields
+    are the serial chain's."""
+    from pdac_amd.gpu import gpu_solver
+    from pdac_amd.solver import PdacError
+    print("[chain fixed point] NaN pressures", flush=True)
+    K_XCHAIN = 19  # PDAC_K_XCHAIN, include/pdacgpu.h
+    out, launches = {}, {}
+    for mode in (None, "general"):
+        chain(monkeypatch, mode)
+        c = eruption_column(nx=24, nz=40, dt=2.0e-4, vent_radius=6.0)
+        c.time_integration = 1
+        g = gpu_solver(c, device=0)
+        p = g.get("p")
+        p.reshape(-1)[3 * c.nx + 3] = np.nan
+        g.put("p", p)
+        for step in range(12):
+            if step == 10:
+                g.lib.pdac_profile_select(g.ctx, 1 << K_XCHAIN)
+                g.lib.pdac_profile_enable(g.ctx, 1)
+                g.lib.pdac_profile_reset(g.ctx)
+            try:
+                g.step(1)
+            except PdacError as e:
+                assert "equation of state" in str(e)
+        n, ms = ct.c_int64(), ct.c_double()
+        assert g.lib.pdac_profile_read(g.ctx, K_XCHAIN, ct.byref(n), ct.byref(ms)) == 0
+        launches[mode] = n.value
+        out[mode] = {k: g.get(k) for k in ("p", "tg", "sieg", "cg", "ug", "rlk")}
+        g.close()
+    print(f"[chain fixed point] chain launches of two steps: {launches}", flush=True)
+    assert np.isnan(out[None]["p"]).any()
+    for k, v in out["general"].items():
+        np.testing.assert_array_equal(out[None][k], v, err_msg=k)
+    # two chained stages a step: a few iterates and two more launches in each
+    assert launches[None] <= 2 * 2 * 20
