@@ -13,9 +13,10 @@
 
 // device counters: sweep state of iter (done flag, sweep numbers of the two
 // colour launches, the sweep that converged), EOS failures, three pairs of
-// unconverged-cell counts per sweep (C_WLP), and for the persistent iteration
-// kernels an arrival counter for grid barriers and an error flag
-enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
+// unconverged-cell counts per sweep (C_WLP), whether a team found no XCD
+// (C_ALONE), and for the persistent iteration kernels an arrival counter for
+// grid barriers and an error flag
+enum Ctr { C_DONE = 0, C_NIT1 = 1, C_NIT = 2, C_ALONE = 3, C_EOS = 4, C_NITF = 5, C_WLP = 8, C_BAR = 14,
            C_ERR = 15, C_N = 16 };
 
 // Words of the sweeps from lists (Fields::team, cleared by k_predict): the

@@ -47,8 +47,8 @@ def solver(case, **env):
             os.environ.pop(k)
 
 
-def run(case, mode, limit=None, steps=3):
-    env = {"PDAC_ITER_MODE": mode}
+def run(case, mode, limit=None, steps=3, **env):
+    env["PDAC_ITER_MODE"] = mode
     if limit:
         env["PDAC_TEAM_LIMIT"] = str(limit)
     g = solver(case, **env)
@@ -103,3 +103,32 @@ def test_long_lists_take_few_attempts():
     assert sweeps > 40 * steps
     assert teams <= 3 * steps
     assert ygas <= 2 * steps
+
+
+@pytest.mark.parametrize("name", ["cone_40", "box_2d_3_classes", "maxout_3"])
+def test_no_compute_units_for_a_team(name):
+    """Fewer blocks than a team needs: the election finds no XCD and gives up
+    after its bounded wait, the call goes on with launches, and later calls do
+    not try again."""
+    print(f"[team] no XCD, {name}", flush=True)
+    a = run(CASES[name](), "team", PDAC_TEAM_GRID="31")
+    b = run(CASES[name](), "launches")
+    assert a[0] == b[0] and a[1] == b[1], (a[:2], b[:2])
+    bad = [k for k in b[2] if not np.array_equal(a[2][k], b[2][k], equal_nan=True)]
+    assert not bad, bad
+    g = solver(CASES[name](), PDAC_TEAM_GRID="31")
+    g.lib.pdac_profile_select(g.ctx, 1 << K_ITERATE)
+    g.lib.pdac_profile_enable(g.ctx, 1)
+    g.lib.pdac_profile_reset(g.ctx)
+    g.step(8)
+    teams = launches(g, K_ITERATE)
+    g.close()
+    # (a launch that finds its lists too long for a team holds no election)
+    assert teams <= 3, teams
+
+
+@pytest.mark.parametrize("value", ["0", "257", "x"])
+def test_team_grid_out_of_range_is_refused(value):
+    from pdac_amd.solver import PdacError
+    with pytest.raises(PdacError, match="PDAC_TEAM_GRID"):
+        solver(CASES["maxout_1"](), PDAC_TEAM_GRID=value)
