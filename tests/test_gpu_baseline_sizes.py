@@ -9,9 +9,9 @@ launch-shape invariance where the checker would take minutes:
   fields to the semi-implicit tolerance;
 - the 3D summit cone with immersed boundaries, 256 x 256 x 192 cells of 10 m,
   three particle classes: two steps in the red-black order against the
-  checker, and five steps in several sweep launch shapes (flag words per
-  thread, list visits between checks, graph replay, the persistent kernel),
-  bit-identical to the default shape;
+  checker, and five steps in several sweep launch shapes (launches with more
+  flag words per thread or list visits between checks, graph replay, the
+  persistent kernel), bit-identical to the default;
 - the explicit eruption column, 256 x 512 uniform 2 m cells: ten steps in the
   reference's cell order, fields to 1e-11 (the explicit step's 1e-12 per
   step, over ten steps)."""
@@ -25,7 +25,7 @@ from pdac_amd import abi
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = ["launches", "launches:12", "launches:24:flush", "launches:7:late", "graph", "persistent"]
+SHAPES = ["team", "team:64", "launches", "launches:12", "launches:24:flush", "launches:7:late", "graph", "persistent"]
 
 
 def rel(a, b):
@@ -36,8 +36,10 @@ def rel(a, b):
     return d / scale if scale > 0.0 else d
 
 
-def gpu(case, mode="launches", **kw):
-    """GPU solver with the sweeps launched as 'mode' says: "launches" (one
+def gpu(case, mode="team", **kw):
+    """GPU solver with the sweeps launched as 'mode' says: "team" (the default:
+    launches while the lists of cells are long, then a team for the remaining
+    sweeps; "team:N" with lists of at most N cells), "launches" (one
     launch per colour phase), "graph" (batches of those replayed as HIP
     graphs), "persistent" (one cooperative kernel); "launches:N" fixes the
     flag words per thread of the 3D sweep kernel, ":late" reads the sweep
@@ -48,7 +50,7 @@ def gpu(case, mode="launches", **kw):
     words, _, order = rest.partition(":")
     env = {"PDAC_ITER_MODE": mode}
     if words:
-        env["PDAC_SWEEP_WORDS"] = words
+        env["PDAC_TEAM_LIMIT" if mode == "team" else "PDAC_SWEEP_WORDS"] = words
     if order == "flush":
         env["PDAC_SWEEP_FLUSH"] = "1"
     elif order:

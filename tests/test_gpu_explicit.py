@@ -125,13 +125,13 @@ def test_stage_order_matches_checker(name):
     assert max(rel(sg[k].reshape(v.shape), v) for k, v in ref.items()) > 1e-10
 
 
-@pytest.mark.parametrize("mode", ["serial", "general"])
-@pytest.mark.parametrize("name", [n for n in EXPLICIT if "_3d" not in n])
+@pytest.mark.parametrize("mode", ["serial", "1"])
+@pytest.mark.parametrize("name", EXPLICIT)
 def test_chain_kernels_match_reference(name, mode, monkeypatch):
     """The default evaluates the reference order's chain as a fixed point of
-    all-cells iterates; the one-lane-per-column serial chain (PDAC_CHAIN=
-    serial, the fallback of the fixed point) and the generic chain kernel
-    (PDAC_CHAIN=general) must give the fixtures' fields as well."""
+    all-cells iterates; the serial chain (PDAC_CHAIN=serial, the last resort of
+    the fixed point) and one iterate with the rest done by one work-group
+    (PDAC_CHAIN=1) must give the fixtures' fields as well."""
     print(f"[explicit chain {mode}] {name}", flush=True)
     monkeypatch.setenv("PDAC_CHAIN", mode)
     case, ref, _ = load(name)

@@ -30,9 +30,11 @@ CONVERGING = [c for c in ALL if c != "mixed_2d_limiters"]
 
 
 def gpu(case, mode="persistent"):
-    """GPU solver; mode selects how the red-black sweeps are launched: all in
+    """GPU solver; mode selects how the red-black sweeps are launched: checks and
+    visits from lists and a team for the remaining sweeps (the default), all in
     one persistent kernel, one launch per colour phase, or batches of such
-    launches replayed as HIP graphs.  "launches:N" also fixes the flag words
+    launches replayed as HIP graphs.  "team:1" lets a team take lists of one
+    cell only, so that launches run most sweeps.  "launches:N" also fixes the flag words
     (4 cells each) each thread of the sweep kernel scans (N = 1..24), which
     the fixtures' small meshes would otherwise leave at one; "launches:N:late" reads the sweep
     counters before the check's first reads, as on meshes too large for a
@@ -45,7 +47,9 @@ def gpu(case, mode="persistent"):
     mode, _, rest = mode.partition(":")
     cpt, _, order = rest.partition(":")
     os.environ["PDAC_ITER_MODE"] = mode
-    if cpt:
+    if mode == "team" and cpt:
+        os.environ["PDAC_TEAM_LIMIT"] = cpt
+    elif cpt:
         os.environ["PDAC_SWEEP_WORDS"] = cpt
     if order == "flush":
         os.environ["PDAC_SWEEP_FLUSH"] = "1"
@@ -54,7 +58,7 @@ def gpu(case, mode="persistent"):
     try:
         return gpu_solver(case, device=0)
     finally:
-        for k in ("PDAC_ITER_MODE", "PDAC_SWEEP_WORDS", "PDAC_SWEEP_EARLY", "PDAC_SWEEP_FLUSH"):
+        for k in ("PDAC_ITER_MODE", "PDAC_TEAM_LIMIT", "PDAC_SWEEP_WORDS", "PDAC_SWEEP_EARLY", "PDAC_SWEEP_FLUSH"):
             os.environ.pop(k, None)
 
 
@@ -89,8 +93,8 @@ STAGES = [
 ]
 
 
-@pytest.mark.parametrize("mode", ["persistent", "launches", "graph", "launches:2", "launches:3", "launches:4",
-                                  "launches:3:late", "launches:7:flush", "launches:24"])
+@pytest.mark.parametrize("mode", ["team", "team:1", "persistent", "launches", "graph", "launches:2", "launches:3",
+                                  "launches:4", "launches:3:late", "launches:7:flush", "launches:24"])
 @pytest.mark.parametrize("name", ALL)
 def test_stagewise(name, mode):
     print(f"[stagewise] {name} {mode}", flush=True)
@@ -174,7 +178,8 @@ def test_fluxes_after_classes_leave(name):
     c.close()
 
 
-@pytest.mark.parametrize("mode", ["persistent", "launches", "graph", "launches:2:late", "launches:5:flush"])
+@pytest.mark.parametrize("mode", ["team", "team:1", "persistent", "launches", "graph", "launches:2:late",
+                                  "launches:5:flush"])
 @pytest.mark.parametrize("name", ALL)
 def test_steps_match_checker(name, mode):
     print(f"[steps] {name} {mode}", flush=True)
@@ -203,11 +208,11 @@ TOL_REF = {"p": 1e-7, "rgp": 2e-7, "rog": 2e-7, "tg": 2e-7, "sieg": 2e-7, "rlk":
 TOL_REF_STIFF = dict(TOL_REF, ug=2e-5, vg=2e-5, wg=2e-5, us=2e-5, vs=2e-5, ws=2e-5)
 
 
-@pytest.mark.parametrize("mode", ["launches", "graph", "launches:2:late", "persistent"])
+@pytest.mark.parametrize("mode", ["team", "team:1", "launches", "graph", "launches:2:late", "persistent"])
 @pytest.mark.parametrize("name", CONVERGING)
 def test_steps_match_reference(name, mode):
-    """Every launch mode of the sweeps (the default, one launch per colour
-    phase, first) against the reference's fixtures."""
+    """Every launch mode of the sweeps (the default, with a team, first) against
+    the reference's fixtures."""
     print(f"[reference] {name} {mode}", flush=True)
     case, ref, nits = load(name)
     g = gpu(case, mode)
@@ -230,8 +235,8 @@ def test_steps_match_reference(name, mode):
 def test_sweep_launch_shapes_agree_on_a_mid_size_cone():
     """The sweep kernel's scan in several launch shapes (flag words per
     thread, so that threads scan several rounds of words; list visits between
-    checks; counters read before or after the first flags; graph replay) and
-    the persistent kernel give the same states bit for bit over three steps of
+    checks; counters read before or after the first flags; graph replay), the
+    persistent kernel and the team give the same states bit for bit over three steps of
     a 64 x 64 x 48 cone with immersed boundaries, a mesh large enough for
     several hundred chunks of flags; the checker in the same order agrees to
     the semi-implicit tolerance."""
@@ -240,7 +245,8 @@ def test_sweep_launch_shapes_agree_on_a_mid_size_cone():
     from pdac_amd.cases import summit_cone_3d
     case = summit_cone_3d(nx=64, ny=64, nz=48, height=375.0, sigma=375.0, rough=7.5, nsteps=1)
     ref, ref_nits, ref_state = None, None, None
-    for mode in ["launches", "launches:12", "launches:12:flush", "launches:5:late", "graph", "persistent"]:
+    for mode in ["launches", "launches:12", "launches:12:flush", "launches:5:late", "graph", "persistent", "team",
+                 "team:1"]:
         print(f"[shapes] {mode}", flush=True)
         g = gpu(case, mode)
         nits = [g.step(1) for _ in range(3)]

@@ -25,6 +25,17 @@ CASES = {
     "box_2d_3_classes": lambda: mixed_box(nx=33, nz=21, nsolid=3, seed=5),
     "vent_odd": lambda: summit_vent_3d(nx=37, ny=41, nz=23, nsolid=2),
     "cone_40": lambda: summit_cone_3d(nx=40, ny=44, nz=30, height=230.0, sigma=230.0, rough=5.0),
+    # the other mass limiters, the other pressure model, no limiter at all
+    "beta": lambda: load("mixed_2d_beta")[0],
+    "variants": lambda: load("mixed_2d_variants")[0],
+    "van_leer_3d": lambda: mixed_box(three_d=True, nx=12, ny=9, nz=10, nsolid=2, mass_limiter=1, maxout=60),
+    "superbee_3d": lambda: mixed_box(three_d=True, nx=12, ny=9, nz=10, nsolid=1, mass_limiter=3, maxout=60),
+    "beta_3d": lambda: mixed_box(three_d=True, nx=9, ny=10, nz=11, nsolid=4, mass_limiter=4, beta=0.3, maxout=60),
+    "ultrabeta_2d": lambda: mixed_box(nx=27, nz=24, nsolid=3, mass_limiter=0, beta=0.3, maxout=60),
+    "pmodel_1_3d": lambda: mixed_box(three_d=True, nx=12, ny=9, nz=10, nsolid=3, pmodel=1),
+    "pmodel_1_one_class": lambda: mixed_box(nx=26, nz=23, nsolid=1, pmodel=1),
+    "muscl_off_2d": lambda: mixed_box(nx=31, nz=22, nsolid=2, muscl=0),
+    "muscl_off_3d": lambda: mixed_box(three_d=True, nx=11, ny=12, nz=9, nsolid=3, muscl=0),
     # lists of a colour up to one round of the whole GPU's waves (2048 cells
     # with three classes in 3D, 1024 with four, 8192 with one class in 2D) and
     # beyond it
