@@ -49,6 +49,9 @@ KERNELS = ["boundary", "fieldn", "momflux", "tilde", "predict", "gasflux", "snap
            "sweep", "ygas_flux", "ygas_update", "htilde_flux", "htilde_update", "ftem", "fill",
            "sweep_check", "iterate", "xinit", "xflux", "xrhs", "xchain", "xmass", "xsolve",
            "stress"]
+# the kernels of the pressure-velocity iteration: checks and visits over the
+# whole GPU, the teams' sweeps, and the scans of the flags before a team
+ITERATION = ("sweep", "iterate", "sweep_check")
 
 
 def words(D, S, G):
@@ -167,7 +170,7 @@ def run_form(args, case, precision, ids):
     # second region of the same length with HIP events around the kernels
     # (events cost host time per launch, so the timed region records none)
     if args.kernel_timing != "none":
-        mask = 0xFFFFFFFF if args.kernel_timing == "all" else (1 << ids["sweep"]) | (1 << ids["iterate"])
+        mask = 0xFFFFFFFF if args.kernel_timing == "all" else sum(1 << ids[k] for k in ITERATION)
         g.lib.pdac_profile_select(g.ctx, mask)
         g.lib.pdac_profile_enable(g.ctx, 1)
     g.lib.pdac_profile_reset(g.ctx)
@@ -428,18 +431,17 @@ def main():
         dom, ms = "none", 0.0
     per_launch_s = ms / 1e3 / max(launches, 1) if launches else float("nan")
     traffic = None
-    if dom in ("sweep", "iterate"):
-        # the kernels of the pressure-velocity iteration together: the checks
-        # and visits over the whole GPU ("sweep") and the team's sweeps
-        # ("iterate").  They read the residual inputs of the cells whose
-        # inputs changed since their last check (check words) and run the
-        # in-cell iteration, which reads and writes the reference sweep's
-        # words of a cell, for those not converged at visit start; the
-        # unchanged cells they skip would give the same result again.  Units
-        # counted on the device over the event region (pdac_profile_checks /
-        # pdac_profile_visits).
+    if dom in ITERATION:
+        # the kernels of the iteration together (a scan of the flags counts in
+        # their time, not as a launch of its own).  They read the residual
+        # inputs of the cells whose inputs changed since their last check
+        # (check words) and run the in-cell iteration, which reads and writes
+        # the reference sweep's words of a cell, for those not converged at
+        # visit start; the unchanged cells they skip would give the same
+        # result again.  Units counted on the device over the event region
+        # (pdac_profile_checks / pdac_profile_visits).
         launches = prof["sweep"][0] + prof["iterate"][0]
-        per_launch_s = (prof["sweep"][1] + prof["iterate"][1]) / 1e3 / launches
+        per_launch_s = sum(prof[k][1] for k in ITERATION) / 1e3 / launches
         dom = "sweep+iterate"
         checks, visits = r["checks"], r["visits"]
         bytes_launch = 8.0 * ((checks - visits) * wc + visits * w["Is"]) / launches

@@ -323,10 +323,12 @@ int pdac_profile_enable(pdac_ctx *ctx, int enable);
 int pdac_profile_select(pdac_ctx *ctx, uint32_t mask);
 int pdac_profile_reset(pdac_ctx *ctx);
 int pdac_profile_read(pdac_ctx *ctx, int kernel, int64_t *launches, double *total_ms);
-/* cells visited by PDAC_K_SWEEP launches (not converged at visit start)
- * since the last pdac_profile_reset */
+/* cells visited by the iteration's launches (PDAC_K_SWEEP, and PDAC_K_ITERATE
+ * where one launch runs several sweeps; PDAC_K_SWEEP_CHECK are the scans of
+ * the flags between the two): cells not converged at visit start, since the
+ * last pdac_profile_reset */
 int pdac_profile_visits(pdac_ctx *ctx, int64_t *visits);
-/* cells whose mass residual PDAC_K_SWEEP launches evaluated (the cells of a
+/* cells whose mass residual those launches evaluated (the cells of a
  * colour phase whose inputs changed since their last check) since the last
  * pdac_profile_reset */
 int pdac_profile_checks(pdac_ctx *ctx, int64_t *checks);
