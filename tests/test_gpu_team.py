@@ -36,13 +36,13 @@ CASES = {
     "pmodel_1_one_class": lambda: mixed_box(nx=26, nz=23, nsolid=1, pmodel=1),
     "muscl_off_2d": lambda: mixed_box(nx=31, nz=22, nsolid=2, muscl=0),
     "muscl_off_3d": lambda: mixed_box(three_d=True, nx=11, ny=12, nz=9, nsolid=3, muscl=0),
-    # lists of a colour up to one round of the whole GPU's waves (2048 cells
-    # with three classes in 3D, 1024 with four, 8192 with one class in 2D) and
-    # beyond it
-    "box_one_round": lambda: mixed_box(three_d=True, nx=18, ny=18, nz=18, nsolid=3),
-    "box_over_a_round": lambda: mixed_box(three_d=True, nx=18, ny=18, nz=19, nsolid=3),
-    "box_4_classes_long": lambda: mixed_box(three_d=True, nx=17, ny=16, nz=15, nsolid=4, seed=7),
-    "box_2d_long": lambda: mixed_box(nx=140, nz=125, nsolid=1),
+    # lists of a colour up to those that k_visit's waves take at two blocks a
+    # compute unit (4096 cells with three classes in 3D, 2048 with four, 16384
+    # with one class in 2D) and beyond them
+    "box_one_round": lambda: mixed_box(three_d=True, nx=34, ny=18, nz=18, nsolid=3),
+    "box_over_a_round": lambda: mixed_box(three_d=True, nx=34, ny=18, nz=19, nsolid=3),
+    "box_4_classes_long": lambda: mixed_box(three_d=True, nx=28, ny=16, nz=15, nsolid=4, seed=7),
+    "box_2d_long": lambda: mixed_box(nx=202, nz=172, nsolid=1),
     "maxout_1": lambda: mixed_box(three_d=True, nx=10, ny=8, nz=9, nsolid=2, maxout=1),
     "maxout_3": lambda: mixed_box(nx=24, nz=18, nsolid=2, maxout=3),
 }
@@ -143,3 +143,27 @@ def test_team_grid_out_of_range_is_refused(value):
     from pdac_amd.solver import PdacError
     with pytest.raises(PdacError, match="PDAC_TEAM_GRID"):
         solver(CASES["maxout_1"](), PDAC_TEAM_GRID=value)
+
+
+def test_two_contexts_in_two_threads():
+    """Two domains stepped at the same time from two threads, each on its own
+    stream: their teams run side by side (or one does without), and each gives
+    what it gives alone."""
+    from concurrent.futures import ThreadPoolExecutor
+    print("[team] two threads", flush=True)
+    names, steps = ("cone_40", "vent_odd"), 12
+    alone = {}
+    for name in names:
+        g = solver(CASES[name]())
+        g.step(steps)
+        alone[name] = (g.nit_total, g.state())
+        g.close()
+    pair = [solver(CASES[name]()) for name in names]
+    with ThreadPoolExecutor(2) as pool:
+        list(pool.map(lambda g: g.step(steps), pair))
+    for name, g in zip(names, pair):
+        nit, st = g.nit_total, g.state()
+        g.close()
+        assert nit == alone[name][0]
+        for k, v in alone[name][1].items():
+            np.testing.assert_array_equal(st[k], v, err_msg=k)
